@@ -724,6 +724,7 @@ int regrow(vpbs_ctx *c, T **p, int64_t n) {
 int lc_buffers(vpbs_ctx *c) {
     const int64_t Np = c->Np;
     if (Np > c->lc_cap) {
+        c->lc_cap = 0;  // until all of them are there
         VPBS_TRY(regrow(c, &c->lc_npos, 3 * Np));
         VPBS_TRY(regrow(c, &c->lc_rec, 12 * Np));
         VPBS_TRY(regrow(c, (NodeSet **)&c->lc_nset, Np));
@@ -743,6 +744,7 @@ int lc_buffers(vpbs_ctx *c) {
 
 int sample_buffers(vpbs_ctx *c, int64_t ns) {
     if (ns > c->lc_cap_s) {
+        c->lc_cap_s = 0;
         VPBS_TRY(regrow(c, &c->lc_sidx, ns));
         VPBS_TRY(regrow(c, &c->lc_spos, 3 * ns));
         c->lc_cap_s = ns;

@@ -982,7 +982,8 @@ int inverse_to_grid(vpbs_ctx *c, Cx<CT> *zp) {
 // Node buffers of the slab interpolation, grown with Np.
 int slab_node_buffers(vpbs_ctx *c) {
     const int64_t Np = c->Np;
-    if (Np <= c->cap_nd && c->nd_key) return VPBS_OK;
+    if (Np <= c->cap_nd) return VPBS_OK;
+    c->cap_nd = 0;  // until all of them are there
     void **bufs[] = {(void **)&c->nd_key, (void **)&c->nd_perm, (void **)&c->nd_i0, (void **)&c->nd_node,
                      &c->nd_rec, &c->slab_part};
     for (void **b : bufs)

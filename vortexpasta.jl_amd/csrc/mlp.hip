@@ -73,9 +73,11 @@ int mfail(vpbs_mlp *m, int code, const char *fmt, ...) {
 #define MLP_HIP(m, expr)                                                                              \
     do {                                                                                              \
         hipError_t e_ = (expr);                                                                       \
-        if (e_ != hipSuccess)                                                                         \
+        if (e_ != hipSuccess) {                                                                       \
+            (void)hipGetLastError(); /* reported here, not by the checks of the next call */          \
             return mfail((m), VPBS_ERR_HIP, "%s failed: %s (%s:%d)", #expr, hipGetErrorString(e_),    \
                          __FILE__, __LINE__);                                                         \
+        }                                                                                             \
     } while (0)
 
 inline unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -457,13 +459,16 @@ int64_t work_floats(const vpbs_mlp *m, int64_t B) {
 
 int ensure_work(vpbs_mlp *m, int64_t B, Work &w) {
     const int64_t need = work_floats(m, B);
+    // a capacity is 0 while its buffer is replaced: an allocation that fails leaves nothing to be taken for valid
     if (need > m->ws_floats) {
+        m->ws_floats = 0;
         if (m->ws) MLP_HIP(m, hipFree(m->ws));
         m->ws = nullptr;
         MLP_HIP(m, hipMalloc((void **)&m->ws, sizeof(float) * (size_t)need));
         m->ws_floats = need;
     }
     if (B > m->cap_idx) {
+        m->cap_idx = 0;
         if (m->idx) MLP_HIP(m, hipFree(m->idx));
         m->idx = nullptr;
         MLP_HIP(m, hipMalloc((void **)&m->idx, sizeof(int32_t) * (size_t)B));
@@ -471,6 +476,7 @@ int ensure_work(vpbs_mlp *m, int64_t B, Work &w) {
     }
     const int64_t nlb = (B * m->n_out + 255) / 256;
     if (nlb > m->cap_loss) {
+        m->cap_loss = 0;
         if (m->loss_part) MLP_HIP(m, hipFree(m->loss_part));
         m->loss_part = nullptr;
         MLP_HIP(m, hipMalloc((void **)&m->loss_part, sizeof(double) * (size_t)nlb));

@@ -777,12 +777,14 @@ int add_local_integrals(vpbs_ctx *c, uint32_t flags, hipStream_t s) {
 int advance_filaments(vpbs_ctx *c, double dt, int nsteps) {
     const int64_t Np = c->Np, n3 = 3 * Np;
     if (n3 > c->cap_step) {
+        c->cap_step = 0;  // until the new buffer is there
         if (c->step_buf) VPBS_HIP(c, hipFree(c->step_buf));
         c->step_buf = nullptr;
         VPBS_HIP(c, hipMalloc((void **)&c->step_buf, sizeof(double) * 2 * (size_t)n3));
         c->cap_step = n3;
     }
     if (12 * Np > c->cap_solve) {
+        c->cap_solve = 0;
         if (c->solve_buf) VPBS_HIP(c, hipFree(c->solve_buf));
         c->solve_buf = nullptr;
         VPBS_HIP(c, hipMalloc((void **)&c->solve_buf, sizeof(double) * 12 * (size_t)Np));

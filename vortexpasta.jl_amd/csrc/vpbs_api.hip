@@ -189,7 +189,12 @@ static int alloc(vpbs_ctx *c, T **p, int64_t n) {
 
 int ensure_capacity(vpbs_ctx *c, int64_t Np, int64_t Nq) {
     const size_t cs = c->p.precision == VPBS_F32 ? sizeof(float) : sizeof(double);
+    if (Np > c->cap_np || Nq > c->cap_nq)  // what the buffers hold goes, also when an allocation fails
+        c->have_points = c->have_filaments = c->have_stats = c->last_vel = c->last_psi = false;
+    // a capacity is 0 while its buffers are replaced: after an allocation that fails the next call, of
+    // whatever size, allocates them all
     if (Np > c->cap_np) {
+        c->cap_np = 0;
         VPBS_TRY(alloc(c, &c->nodes, 3 * Np));
         VPBS_TRY(alloc(c, &c->sp, 3 * Np));
         VPBS_TRY(alloc(c, &c->spp, 3 * Np));
@@ -211,6 +216,7 @@ int ensure_capacity(vpbs_ctx *c, int64_t Np, int64_t Nq) {
         c->cap_np = Np;
     }
     if (Nq > c->cap_nq) {
+        c->cap_nq = 0;
         VPBS_TRY(alloc(c, &c->points, 3 * Nq));
         VPBS_TRY(alloc(c, &c->charges, 3 * Nq));
         VPBS_TRY(alloc(c, &c->src_key, Nq));

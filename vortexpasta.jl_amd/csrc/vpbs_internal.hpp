@@ -256,9 +256,11 @@ int fail(vpbs_ctx *c, int code, const char *fmt, ...);
 #define VPBS_HIP(ctx, expr)                                                                        \
     do {                                                                                           \
         hipError_t e_ = (expr);                                                                    \
-        if (e_ != hipSuccess)                                                                      \
+        if (e_ != hipSuccess) {                                                                    \
+            (void)hipGetLastError(); /* reported here, not by the checks of the next call */       \
             return ::vpbs::fail((ctx), VPBS_ERR_HIP, "%s failed: %s (%s:%d)", #expr,               \
                                 hipGetErrorString(e_), __FILE__, __LINE__);                        \
+        }                                                                                          \
     } while (0)
 
 #define VPBS_TRY(expr)          \
