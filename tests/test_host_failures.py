@@ -43,6 +43,13 @@ def test_out_of_memory_while_growing(fake_hip, work):
         assert all(a >= b for a, b in zip(after["blocks"], out["fresh"])), f"allocation {k}: buffers too small"
 
 
+@pytest.mark.parametrize("call", ["hipHostGetDevicePointer", "hipLaunchKernel"])
+def test_filaments_are_there_once_their_kernels_ran(fake_hip, call):
+    """An upload that fails before its kernels ran leaves no filaments to step: the filament of each node, which the
+    step's kernels index with, comes from them."""
+    assert run(fake_hip, "upload", call) == {"upload": True, "advance": True, "again": ""}
+
+
 # --------------------------------------------------------------------------- #
 # In the process of its own
 
@@ -88,13 +95,16 @@ class Work:
             s.set_points(points(n))
             s.compute(F.VELOCITY | F.STREAMFUNCTION | F.KEEP_UHAT | F.NEIGHBOUR_STATS)
             return s.energy_spectrum(max(n // 10, 1), 1.0)
-        t = TWO_PI * np.arange(n) / n
-        X = np.stack([1 + np.cos(t), 2 + np.sin(t), 3 + 0.1 * np.sin(3 * t)], axis=1)
-        s.set_filaments(self.vp.FilamentBatch([self.vp.ClosedFilament(X, np.zeros(3))]), self.p)
+        self.upload(s, n)
         if self.kind == "learned":
             s.compute_learned()
         else:
             s.advance(1e-3, 1)
+
+    def upload(self, s, n):
+        t = TWO_PI * np.arange(n) / n
+        X = np.stack([1 + np.cos(t), 2 + np.sin(t), 3 + 0.1 * np.sin(3 * t)], axis=1)
+        s.set_filaments(self.vp.FilamentBatch([self.vp.ClosedFilament(X, np.zeros(3))]), self.p)
 
     def stale(self, s):
         """Calls on what the failed one replaced, of which none may find anything."""
@@ -156,15 +166,40 @@ def grow_and_fail(vp, fake, kind):
     return out
 
 
+def upload_and_fail(vp, fake, call):
+    w = Work(vp, "advance")
+    s = w.start()
+    out = {}
+
+    def refused(f):
+        try:
+            f()
+        except vp._lib.VpbsError as e:
+            return str(e)
+        return ""
+
+    fake.fake_fail_call(call.encode())
+    out["upload"] = "invalid value" in refused(lambda: w.upload(s, 60))
+    fake.fake_fail_call(None)
+    out["advance"] = "no filaments on the device" in refused(lambda: s.advance(1e-3, 1))
+    out["again"] = refused(lambda: w.call(s, 60))
+    s.close()
+    return out
+
+
 def main():
     fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
     fake.fake_mallocs.restype = fake.fake_launches.restype = ctypes.c_long
     fake.fake_fail_malloc.argtypes = [ctypes.c_long]
+    fake.fake_fail_call.argtypes = [ctypes.c_char_p]
     sys.path.insert(0, str(HERE.parent))
     import __graft_entry__ as ge
 
     vp = ge.load_package()
-    print(json.dumps(grow_and_fail(vp, fake, sys.argv[2])))
+    if sys.argv[2] == "upload":
+        print(json.dumps(upload_and_fail(vp, fake, sys.argv[3])))
+    else:
+        print(json.dumps(grow_and_fail(vp, fake, sys.argv[2])))
 
 
 if __name__ == "__main__":

@@ -629,6 +629,7 @@ int point_data_from_state(vpbs_ctx *c, bool uploaded) {
     VPBS_HIP(c, hipGetLastError());
     stage_end(c, ST_POINTS, s);
     VPBS_HIP(c, hipStreamSynchronize(s));
+    c->have_filaments = true;  // complete from here on: the filament of each node comes from the first kernel
     if (*flag) VPBS_TRY(device_check(c));  // counts what is wrong
     float ms = 0.f;
     VPBS_HIP(c, hipEventElapsedTime(&ms, c->stage_from[ST_POINTS], c->ev_end[ST_POINTS]));
@@ -747,7 +748,6 @@ int build_point_data(vpbs_ctx *c, int64_t Nf, const int64_t *counts, const doubl
     }
     c->Np = Np;
     c->Nq = Nq;
-    c->have_filaments = true;
     return point_data_from_state(c, true);
 }
 
