@@ -158,7 +158,7 @@ __device__ inline int64_t gather_record(int64_t t, int64_t n, const int32_t *key
     constexpr int M = W / 2;
     j = perm[t];
     const int32_t b = key[j];
-    const int64_t s = bin_place(perm, start[b], start[b + 1], j);
+    const int64_t s = bin_place(perm, n, start[b], start[b + 1], j, (int32_t)t);
     CT r[REC];
 #pragma unroll
     for (int k = 3 * W; k < REC; k++) r[k] = (CT)0;
@@ -1014,8 +1014,8 @@ int launch_lr(vpbs_ctx *c, uint32_t flags) {
     stage_begin(c, ST_LRSORT, s);
     if (c->slab_interp) VPBS_TRY(slab_node_buffers(c));
     BinList lists[2] = {
-        {BIN_TILE, Nq, c->ntiles, c->points, c->lr_key, c->lr_start, c->lr_perm, nullptr},
-        {BIN_SLAB, Np, c->nslabs, c->nodes, c->nd_key, c->nd_start, c->nd_perm, nullptr},
+        {BIN_TILE, Nq, c->ntiles, c->points, c->lr_key, c->lr_start, c->lr_perm, nullptr, true},
+        {BIN_SLAB, Np, c->nslabs, c->nodes, c->nd_key, c->nd_start, c->nd_perm, nullptr, true},
     };
     VPBS_TRY(bin_lists(c, c->sort_lr, lists, c->slab_interp ? 2 : 1, s));
     GatherArgs<CT> ga{g, beta, Nq, Np, nblocks(Nq, 256), c->lr_key, c->lr_start, c->lr_perm, c->nd_key, c->nd_start,

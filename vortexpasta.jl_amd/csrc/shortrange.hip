@@ -85,7 +85,7 @@ __global__ void gather_sources(int64_t Nq, const int32_t *__restrict__ key, cons
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= Nq) return;
     const int32_t j = perm[t], k = key[j];
-    const int64_t s = bin_place(perm, start[k], start[k + 1], j);
+    const int64_t s = bin_place(perm, 0, start[k], start[k + 1], j, (int32_t)t);
     sidx[s] = j;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
@@ -806,12 +806,14 @@ int run_pairs(vpbs_ctx *c, bool vel, bool psi, bool stats, bool include_local) {
     hipStream_t s = c->s_sr;
     const int3 Nc = make_int3(c->Nc[0], c->Nc[1], c->Nc[2]);
     stage_begin(c, ST_CELL, s);
+    // Large cells are ordered by counting as well: the pair sum of a cell is quadratic in its population
+    // too, ten times as much (100k sources and nodes in one cell: 2.9 and 33 ms).
     // The nodes keep the order of the atomic ranks inside a cell: the pair kernel's sums do not
     // depend on it (it only sets the processing order), and the feature kernel breaks distance
     // ties by node index.
     BinList lists[2] = {
-        {BIN_CELL, Nq, c->ncells, c->points, c->src_key, c->src_start, c->src_perm, nullptr},
-        {BIN_CELL, Np, c->ncells, c->nodes, c->tgt_key, c->tgt_start, c->tgt_perm, c->tgt_cell},
+        {BIN_CELL, Nq, c->ncells, c->points, c->src_key, c->src_start, c->src_perm, nullptr, false},
+        {BIN_CELL, Np, c->ncells, c->nodes, c->tgt_key, c->tgt_start, c->tgt_perm, c->tgt_cell, false},
     };
     VPBS_TRY(bin_lists(c, c->sort_sr, lists, 2, s));
     gather_sources<CT><<<nblocks(Nq, 256), 256, 0, s>>>(Nq, c->src_key, c->src_start, c->src_perm, c->points,

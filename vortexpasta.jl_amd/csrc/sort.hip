@@ -11,6 +11,7 @@
 //   3. sums of 2048-bin tiles, then an exclusive scan of each tile on top of the sums
 //      before it
 //   4. scatter to start[key] + rank
+//   5. tiles and slabs: a block per large bin (bin_large; found by the scan) puts it in order
 //
 // The order inside a bin is then that of the arrival ranks. The kernels that gather the
 // binned data put an element at start + (number of smaller indices in its bin) (bin_place
@@ -22,10 +23,14 @@
 // sorted only to find the bins again. Why no sort of each bin's segment: one thread per bin
 // took 160-450 us wherever a few bins hold most points. Five launches for both lists; points
 // and nodes of 256k nodes, LR stream, 0.21 -> 0.11 ms; cell lists 0.20 -> 0.07 ms. The count of
-// smaller indices is quadratic in a bin's population, but so (with a larger constant) is the
-// pair sum of a cell, and a tile's or slab's population is walked by one block afterwards.
+// smaller indices is quadratic in a bin's population, while the walks over a tile or a slab that come
+// after are linear: large tiles and slabs are put in order by step 5 instead. Sort and records on 384³
+// cells, all points and nodes in one tile and slab: 100k 3.3 -> 0.24 ms, 1M 219 -> 4.7 ms (the radix sort
+// 1.7 and 2.0); on lines along x in one slab: 1M 117 -> 6.4 ms.
 #include "vpbs_internal.hpp"
 #include "device_util.hpp"
+
+#include <algorithm>
 
 namespace vpbs {
 
@@ -75,6 +80,7 @@ __device__ inline int list_of(const BinGroup &g, const unsigned (&first)[2]) {
 __global__ __launch_bounds__(256) void bin_zero(BinGroup g) {
     const int t = list_of(g, g.scan_block);
     const BinList &l = g.l[t];
+    if (g.large && blockIdx.x == 0 && threadIdx.x == 0) g.large[0] = 0;
     const int64_t base = (int64_t)(blockIdx.x - g.scan_block[t]) * SCAN_TILE + threadIdx.x;
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
@@ -131,9 +137,9 @@ __global__ __launch_bounds__(SCAN_BS) void bin_tile_sums(BinGroup g) {
 }
 
 // Exclusive scan of one tile in place, on top of what comes before it: the sums of the tiles
-// before it added up here, or (scanned) read from their exclusive scan.
+// before it added up here, or (scanned) read from their exclusive scan. Large bins go to `large`.
 __device__ inline void scan_tile(int32_t *a, int64_t n, int64_t tile, const int32_t *sums, bool scanned, int32_t *s_tot,
-                                 int32_t *s_tot2) {
+                                 int32_t *s_tot2, int32_t *large = nullptr, int list = 0, int64_t elements = 0) {
     int32_t before = 0;
     if (scanned) {
         before = sums[tile];
@@ -159,6 +165,11 @@ __device__ inline void scan_tile(int32_t *a, int64_t n, int64_t tile, const int3
     for (int k = 0; k < SCAN_IPT; k++) {
         if (base + k < n) a[base + k] = run;
         run += v[k];
+        if (large && bin_large(elements, v[k])) {
+            const int e = atomicAdd(large, 1);
+            large[1 + 2 * e] = list;
+            large[2 + 2 * e] = (int32_t)(base + k);
+        }
     }
 }
 
@@ -166,7 +177,8 @@ __global__ __launch_bounds__(SCAN_BS) void bin_scan(BinGroup g, int scanned) {
     __shared__ int32_t s_tot[SCAN_BS / 64], s_tot2[SCAN_BS / 64];
     const int t = list_of(g, g.scan_block);
     const BinList &l = g.l[t];
-    scan_tile(l.start, l.nbins + 1, blockIdx.x - g.scan_block[t], l.sums, scanned != 0, s_tot, s_tot2);
+    scan_tile(l.start, l.nbins + 1, blockIdx.x - g.scan_block[t], l.sums, scanned != 0, s_tot, s_tot2,
+              l.order_large ? g.large : nullptr, t, l.n);
 }
 
 // Levels of a scan with more than SCAN_FLAT_TILES tiles.
@@ -205,6 +217,66 @@ __global__ __launch_bounds__(256) void bin_scatter(BinGroup g) {
     if (j < l.n) l.perm[l.start[l.key[j]] + l.rank[j]] = (int32_t)j;
 }
 
+// Large bins, one block each: the bin's elements as bits of a window of indices in LDS, window after
+// window; the set bits, in order, are the bin in order (through the ranks, which are done with). Linear in
+// the bin's population per window of 131072 indices, bound by the latency of its loads. Blocks small
+// enough to start beside the other stream's kernels: usually there is nothing to do (blocks of 1024
+// threads with 33 KB made a call of 1.14 ms 3 % slower).
+constexpr int ORDER_NT = 256, ORDER_WORDS = 16 * ORDER_NT, ORDER_WINDOW = 32 * ORDER_WORDS;
+constexpr int64_t ORDER_BLOCKS = 256;
+__global__ __launch_bounds__(ORDER_NT) void bin_order(BinGroup g) {
+    __shared__ uint32_t bits[ORDER_WORDS];
+    __shared__ int32_t s_tot[ORDER_NT / 64];
+    constexpr int PER = ORDER_WORDS / ORDER_NT;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int count = g.large[0];
+    for (int e = blockIdx.x; e < count; e += gridDim.x) {
+        const BinList &l = g.l[g.large[1 + 2 * e]];
+        const int32_t bin = g.large[2 + 2 * e], s0 = l.start[bin], s1 = l.start[bin + 1];
+        const int32_t v0 = (s0 + 3) & ~3, v1 = s1 & ~3;  // whole 16-byte vectors (population > BIN_LARGE: v0 < v1)
+        int32_t at = s0;
+        for (int64_t first = 0; first < l.n && at < s1; first += ORDER_WINDOW) {
+#pragma unroll
+            for (int q = 0; q < PER; q++) bits[threadIdx.x + q * ORDER_NT] = 0;
+            __syncthreads();
+            auto set = [&](int32_t j) {
+                const uint32_t i = (uint32_t)j - (uint32_t)first;
+                if (i < (uint32_t)ORDER_WINDOW) atomicOr(&bits[i >> 5], 1u << (i & 31));
+            };
+#pragma unroll 4
+            for (int32_t k = v0 + 4 * (int32_t)threadIdx.x; k < v1; k += 4 * ORDER_NT) {
+                const int4 v = *reinterpret_cast<const int4 *>(l.perm + k);
+                set(v.x), set(v.y), set(v.z), set(v.w);
+            }
+            if (s0 + (int32_t)threadIdx.x < v0) set(l.perm[s0 + threadIdx.x]);
+            if (v1 + (int32_t)threadIdx.x < s1) set(l.perm[v1 + threadIdx.x]);
+            __syncthreads();
+            uint32_t b[PER];
+            int n = 0;
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                b[q] = bits[PER * threadIdx.x + q];
+                n += __popc(b[q]);
+            }
+            const int incl = wave_incl_scan(n);
+            if (lane == 63) s_tot[wid] = incl;
+            __syncthreads();
+            int32_t to = at + incl - n;
+#pragma unroll
+            for (int w = 0; w < ORDER_NT / 64; w++) {
+                to += w < wid ? s_tot[w] : 0;
+                at += s_tot[w];
+            }
+#pragma unroll
+            for (int q = 0; q < PER; q++)
+                for (uint32_t m = b[q]; m; m &= m - 1)
+                    l.rank[to++] = (int32_t)first + 32 * (PER * (int32_t)threadIdx.x + q) + __ffs(m) - 1;
+            __syncthreads();  // bits and sums are read, the ranks written
+        }
+        for (int32_t k = s0 + (int32_t)threadIdx.x; k < s1; k += ORDER_NT) l.perm[k] = l.rank[k];
+    }
+}
+
 // Storage of the tile sums of n values and of every level above them.
 int64_t sums_size(int64_t n) {
     int64_t tot = 1;
@@ -228,13 +300,18 @@ int bin_lists(vpbs_ctx *c, SortBuffers &sb, BinList *lists, int count, hipStream
         g.geom.G[d] = c->G[d];
         g.geom.scale[d] = (double)c->G[d] / c->p.Ls[d];
     }
-    int64_t n = 0, nsum = 0;
+    int64_t n = 0, nsum = 0, nlarge = 0;  // nlarge: at most
     for (int t = 0; t < count; t++) {
         n += lists[t].n;
         nsum += sums_size(lists[t].nbins + 1);
+        if (lists[t].order_large && bin_large(lists[t].n, lists[t].n)) nlarge += lists[t].n / (BIN_LARGE + 1);
     }
     VPBS_TRY(grow(c, &sb.rank, &sb.cap_n, n));
     VPBS_TRY(grow(c, &sb.sums, &sb.cap_sums, nsum));
+    if (nlarge) {
+        VPBS_TRY(grow(c, &sb.large, &sb.cap_large, 1 + 2 * nlarge));
+        g.large = sb.large;
+    }
     unsigned eb = 0, tb = 0;
     int32_t *rank = sb.rank, *sums = sb.sums;
     bool deep = false;
@@ -262,6 +339,7 @@ int bin_lists(vpbs_ctx *c, SortBuffers &sb, BinList *lists, int count, hipStream
         }
     bin_scan<<<tb, SCAN_BS, 0, s>>>(g, deep);
     bin_scatter<<<eb, 256, 0, s>>>(g);
+    if (nlarge) bin_order<<<(unsigned)std::min(nlarge, ORDER_BLOCKS), ORDER_NT, 0, s>>>(g);
     VPBS_HIP(c, hipGetLastError());
     return VPBS_OK;
 }

@@ -160,7 +160,8 @@ static void release(vpbs_ctx *c) {
                     c->v_out,     c->psi_out,   c->src_key,  c->src_start, c->src_perm,   c->tgt_key,   c->tgt_cell,
                     c->tgt_start, c->tgt_perm,  c->src_pos,  c->src_chg,   c->src_idx,    c->stat_counts, c->stat_cands,
                     c->stat_hashes, c->lr_key,  c->lr_start, c->lr_perm,   c->lr_i0,      c->lr_w,
-                    c->sort_sr.rank, c->sort_sr.sums, c->sort_lr.rank, c->sort_lr.sums,
+                    c->sort_sr.rank, c->sort_sr.sums, c->sort_sr.large, c->sort_lr.rank, c->sort_lr.sums,
+                    c->sort_lr.large,
                     c->nd_key,    c->nd_start,  c->nd_perm,  c->nd_i0,    c->nd_node,    c->nd_rec,     c->slab_part,
                     c->fil_block, c->fil_d,   c->fil_e,   c->fil_fid, c->step_buf,    c->solve_buf,
                     c->check_dev, c->spec_part};

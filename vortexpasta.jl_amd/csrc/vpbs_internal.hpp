@@ -18,12 +18,14 @@ struct Box {
     double Lh[3];
 };
 
-// Scratch of bin_lists (grow-only device buffers): arrival ranks, then sums of histogram tiles.
+// Scratch of bin_lists (grow-only device buffers): arrival ranks, sums of histogram tiles, large bins.
 struct SortBuffers {
     int32_t *rank = nullptr;
     int64_t cap_n = 0;
     int32_t *sums = nullptr;
     int64_t cap_sums = 0;
+    int32_t *large = nullptr;  // number of large bins, then (list, bin) of each
+    int64_t cap_large = 0;
 };
 
 // Slabs of the interpolation fused with the inverse x transform: SLAB_HY y-rows × slab_hz z-rows ×
@@ -40,6 +42,15 @@ constexpr int SPREAD_TX = 16, SPREAD_TY = 8, SPREAD_TZ = 8;
 // A list of positions to bin (sort.hip): by cell of the short-range cell lists, or by the
 // spreading tile or the slab of the first stencil cell.
 enum BinKind { BIN_CELL, BIN_TILE, BIN_SLAB };
+// Whether a bin of a list of n elements is put in order by a block of its own (bin_order in sort.hip) and
+// not by counting. Sort and records of one bin of 600 points and nodes take 52 µs so and 47 by counting,
+// of 1000 56 and 62, of 2000 62 and 91, of 8000 70 and 277. In short lists counting costs at most 0.5 ms
+// (all elements in one bin), and the launch, 5 µs of every call, is left out.
+constexpr int BIN_LARGE = 768;
+constexpr int64_t BIN_SHORT_LIST = 16384;
+__host__ __device__ constexpr bool bin_large(int64_t n, int64_t population) {
+    return n > BIN_SHORT_LIST && population > BIN_LARGE;
+}
 struct BinList {
     int kind;
     int64_t n, nbins;
@@ -48,6 +59,7 @@ struct BinList {
     int32_t *start;     // out: start[b] = first place of bin b, start[nbins] = n
     int32_t *perm;      // out: the elements of every bin, in any order inside it
     int32_t *cell;      // out, or null: per element (ix, iy, iz, key) of its cell
+    bool order_large;   // large bins in order of index
     int32_t *rank = nullptr, *sums = nullptr;  // scratch
 };
 struct BinGeom {
@@ -59,6 +71,7 @@ struct BinGroup {
     int count;
     BinList l[2];
     unsigned elem_block[2], scan_block[2];  // first block of each list
+    int32_t *large;                         // null: there can be none to put in order
     BinGeom geom;
 };
 // Node record of that interpolation: the W kernel weights per direction, padded to
