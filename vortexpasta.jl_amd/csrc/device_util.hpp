@@ -86,12 +86,9 @@ __device__ inline int wave_incl_max(int v) {
     return v;
 }
 
-// Place of element j = perm[t] in the order (bin, index): its bin's start plus the smaller indices in
-// the bin, or t in the large bins of a list of n whose large bins bin_lists orders (n = 0: it does not).
-// perm, start as bin_lists leaves them; s0 = start[bin], s1 = start[bin + 1].
-__device__ inline int32_t bin_place(const int32_t *__restrict__ perm, int64_t n, int32_t s0, int32_t s1, int32_t j,
-                                    int32_t t) {
-    if (bin_large(n, s1 - s0)) return t;
+// Place of element j in the order (bin, index): its bin's start plus the smaller indices in the bin
+// (perm, start as bin_lists leaves them; s0 = start[bin], s1 = start[bin + 1]).
+__device__ inline int32_t bin_place(const int32_t *__restrict__ perm, int32_t s0, int32_t s1, int32_t j) {
     int32_t r = s0, k = s0;
     for (; k < s1 && (k & 3); k++) r += perm[k] < j ? 1 : 0;
     for (; k + 4 <= s1; k += 4) {

@@ -153,12 +153,16 @@ __device__ __forceinline__ void load_rec(const CT *__restrict__ p, CT (&r)[N]) {
 // returned with the element in j.
 template <typename CT, int W, int REC>
 __device__ inline int64_t gather_record(int64_t t, int64_t n, const int32_t *key, const int32_t *start,
-                                        const int32_t *perm, const double *pos, const double *chg, const LRGeom &g,
+                                        const int32_t *perm, const int32_t *ordered, const double *pos, const double *chg, const LRGeom &g,
                                         CT beta, int32_t *si0, CT *rec, int32_t &j) {
     constexpr int M = W / 2;
     j = perm[t];
-    const int32_t b = key[j];
-    const int64_t s = bin_place(perm, n, start[b], start[b + 1], j, (int32_t)t);
+    const int32_t b = key[j], s0 = start[b], s1 = start[b + 1];
+    int64_t s = t;
+    if (bin_large(n, s1 - s0))
+        j = ordered[t];
+    else
+        s = bin_place(perm, s0, s1, j);
     CT r[REC];
 #pragma unroll
     for (int k = 3 * W; k < REC; k++) r[k] = (CT)0;
@@ -181,7 +185,7 @@ struct GatherArgs {
     CT beta;
     int64_t Nq, Np;
     unsigned point_blocks;  // blocks of 256 points, followed by blocks of 256 nodes
-    const int32_t *pkey, *pstart, *pperm, *nkey, *nstart, *nperm;
+    const int32_t *pkey, *pstart, *pperm, *pordered, *nkey, *nstart, *nperm, *nordered;
     const double *pts, *chg, *nodes;
     int32_t *pi0, *ni0, *nnode;  // nnode: node of each slab-sorted place
     CT *prec, *nrec;
@@ -195,12 +199,12 @@ __global__ __launch_bounds__(256) void gather_records(GatherArgs<CT> a) {
     if (blockIdx.x < a.point_blocks) {
         const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
         if (t >= a.Nq) return;
-        gather_record<CT, W, rec_len(W)>(t, a.Nq, a.pkey, a.pstart, a.pperm, a.pts, a.chg, a.g, a.beta, a.pi0, a.prec, j);
+        gather_record<CT, W, rec_len(W)>(t, a.Nq, a.pkey, a.pstart, a.pperm, a.pordered, a.pts, a.chg, a.g, a.beta, a.pi0, a.prec, j);
     } else {
         const int64_t t = (int64_t)(blockIdx.x - a.point_blocks) * 256 + threadIdx.x;
         if (t >= a.Np) return;
         const int64_t s = gather_record<CT, W, slab_rec_len(W, (int)sizeof(CT))>(
-            t, a.Np, a.nkey, a.nstart, a.nperm, a.nodes, nullptr, a.g, a.beta, a.ni0, a.nrec, j);
+            t, a.Np, a.nkey, a.nstart, a.nperm, a.nordered, a.nodes, nullptr, a.g, a.beta, a.ni0, a.nrec, j);
         a.nnode[s] = j;
     }
 }
@@ -1018,8 +1022,8 @@ int launch_lr(vpbs_ctx *c, uint32_t flags) {
         {BIN_SLAB, Np, c->nslabs, c->nodes, c->nd_key, c->nd_start, c->nd_perm, nullptr, true},
     };
     VPBS_TRY(bin_lists(c, c->sort_lr, lists, c->slab_interp ? 2 : 1, s));
-    GatherArgs<CT> ga{g, beta, Nq, Np, nblocks(Nq, 256), c->lr_key, c->lr_start, c->lr_perm, c->nd_key, c->nd_start,
-                      c->nd_perm, c->points, c->charges, c->nodes, c->lr_i0, c->nd_i0, c->nd_node, (CT *)c->lr_w,
+    GatherArgs<CT> ga{g, beta, Nq, Np, nblocks(Nq, 256), c->lr_key, c->lr_start, c->lr_perm, lists[0].rank, c->nd_key,
+                      c->nd_start, c->nd_perm, lists[1].rank, c->points, c->charges, c->nodes, c->lr_i0, c->nd_i0, c->nd_node, (CT *)c->lr_w,
                       (CT *)c->nd_rec};
     launch_gather<CT>(ga, ga.point_blocks + (c->slab_interp ? nblocks(Np, 256) : 0), s);
     stage_end(c, ST_LRSORT, s);

@@ -85,7 +85,7 @@ __global__ void gather_sources(int64_t Nq, const int32_t *__restrict__ key, cons
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= Nq) return;
     const int32_t j = perm[t], k = key[j];
-    const int64_t s = bin_place(perm, 0, start[k], start[k + 1], j, (int32_t)t);
+    const int64_t s = bin_place(perm, start[k], start[k + 1], j);
     sidx[s] = j;
 #pragma unroll
     for (int d = 0; d < 3; d++) {

@@ -11,7 +11,7 @@
 //   3. sums of 2048-bin tiles, then an exclusive scan of each tile on top of the sums
 //      before it
 //   4. scatter to start[key] + rank
-//   5. tiles and slabs: a block per large bin (bin_large; found by the scan) puts it in order
+//   5. tiles and slabs: blocks for every large bin (bin_large; found by the scan) put it in order
 //
 // The order inside a bin is then that of the arrival ranks. The kernels that gather the
 // binned data put an element at start + (number of smaller indices in its bin) (bin_place
@@ -25,8 +25,8 @@
 // and nodes of 256k nodes, LR stream, 0.21 -> 0.11 ms; cell lists 0.20 -> 0.07 ms. The count of
 // smaller indices is quadratic in a bin's population, while the walks over a tile or a slab that come
 // after are linear: large tiles and slabs are put in order by step 5 instead. Sort and records on 384³
-// cells, all points and nodes in one tile and slab: 100k 3.3 -> 0.24 ms, 1M 219 -> 4.7 ms (the radix sort
-// 1.7 and 2.0); on lines along x in one slab: 1M 117 -> 6.4 ms.
+// cells, all points and nodes in one tile and slab: 100k 3.3 -> 0.15 ms, 1M 219 -> 0.93 ms (the radix sort
+// 1.7 and 2.0); on lines along x in one slab: 1M 117 -> 2.3 ms (2.2).
 #include "vpbs_internal.hpp"
 #include "device_util.hpp"
 
@@ -98,15 +98,30 @@ __global__ __launch_bounds__(256) void bin_histogram(BinGroup g) {
     // runs of equal keys: the first lane of each adds the run's length
     const int32_t prev = __shfl_up(key, 1, 64);
     const unsigned long long heads = __ballot(lane == 0 || key != prev);
-    const int first = 63 - __clzll(heads & (~0ull >> (63 - lane)));
+    int first = 63 - __clzll(heads & (~0ull >> (63 - lane)));
     const unsigned long long later = heads & ~(~0ull >> (63 - first));  // heads of later runs
-    const int end = later ? __ffsll(later) - 1 : 64;
+    int count = (later ? __ffsll(later) - 1 : 64) - first, place = lane - first;
+    // the runs of up to four keys together: elements in no order, few bins (a million atomics on one
+    // counter take 3 ms)
+    unsigned long long todo = heads;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        if (!todo) break;
+        const int lead = __ffsll(todo) - 1;
+        const unsigned long long same = __ballot(key == __builtin_amdgcn_readlane(key, lead));
+        if (same >> lane & 1) {
+            first = lead;
+            count = __popcll(same);
+            place = __popcll(same & ((1ull << lane) - 1ull));
+        }
+        todo &= ~same;
+    }
     int base = 0;
-    if (lane == first && key >= 0) base = atomicAdd(&l.start[key], end - first);
+    if (lane == first && key >= 0) base = atomicAdd(&l.start[key], count);
     base = __shfl(base, first, 64);
     if (j < l.n) {
         l.key[j] = key;
-        l.rank[j] = base + (lane - first);
+        l.rank[j] = base + place;
     }
 }
 
@@ -217,63 +232,63 @@ __global__ __launch_bounds__(256) void bin_scatter(BinGroup g) {
     if (j < l.n) l.perm[l.start[l.key[j]] + l.rank[j]] = (int32_t)j;
 }
 
-// Large bins, one block each: the bin's elements as bits of a window of indices in LDS, window after
-// window; the set bits, in order, are the bin in order (through the ranks, which are done with). Linear in
-// the bin's population per window of 131072 indices, bound by the latency of its loads. Blocks small
-// enough to start beside the other stream's kernels: usually there is nothing to do (blocks of 1024
-// threads with 33 KB made a call of 1.14 ms 3 % slower).
+// Large bins: a block per bin and window of indices marks the bin's elements in the window as bits in LDS
+// and writes the set bits, in order, behind the bin's smaller elements (into the ranks, which are done
+// with). Bound by the latency of the loads; the blocks are small enough to start beside the other
+// stream's kernels, since usually there is nothing to do (blocks of 1024 threads with 33 KB made a call of
+// 1.14 ms 3 % slower).
 constexpr int ORDER_NT = 256, ORDER_WORDS = 16 * ORDER_NT, ORDER_WINDOW = 32 * ORDER_WORDS;
-constexpr int64_t ORDER_BLOCKS = 256;
-__global__ __launch_bounds__(ORDER_NT) void bin_order(BinGroup g) {
+constexpr int64_t ORDER_BLOCKS = 1024;
+__global__ __launch_bounds__(ORDER_NT) void bin_order(BinGroup g, int windows) {
     __shared__ uint32_t bits[ORDER_WORDS];
-    __shared__ int32_t s_tot[ORDER_NT / 64];
+    __shared__ int32_t s_tot[ORDER_NT / 64], s_before[ORDER_NT / 64];
     constexpr int PER = ORDER_WORDS / ORDER_NT;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int count = g.large[0];
-    for (int e = blockIdx.x; e < count; e += gridDim.x) {
+    const int64_t items = (int64_t)g.large[0] * windows;
+    for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+        const int e = (int)(item / windows);
+        const int64_t first = (item - (int64_t)e * windows) * ORDER_WINDOW;
         const BinList &l = g.l[g.large[1 + 2 * e]];
+        if (first >= l.n) continue;
         const int32_t bin = g.large[2 + 2 * e], s0 = l.start[bin], s1 = l.start[bin + 1];
         const int32_t v0 = (s0 + 3) & ~3, v1 = s1 & ~3;  // whole 16-byte vectors (population > BIN_LARGE: v0 < v1)
-        int32_t at = s0;
-        for (int64_t first = 0; first < l.n && at < s1; first += ORDER_WINDOW) {
 #pragma unroll
-            for (int q = 0; q < PER; q++) bits[threadIdx.x + q * ORDER_NT] = 0;
-            __syncthreads();
-            auto set = [&](int32_t j) {
-                const uint32_t i = (uint32_t)j - (uint32_t)first;
-                if (i < (uint32_t)ORDER_WINDOW) atomicOr(&bits[i >> 5], 1u << (i & 31));
-            };
+        for (int q = 0; q < PER; q++) bits[threadIdx.x + q * ORDER_NT] = 0;
+        __syncthreads();
+        int before = 0;
+        auto set = [&](int32_t j) {
+            const uint32_t i = (uint32_t)j - (uint32_t)first;
+            if (i < (uint32_t)ORDER_WINDOW) atomicOr(&bits[i >> 5], 1u << (i & 31));
+            before += j < (int32_t)first ? 1 : 0;
+        };
 #pragma unroll 4
-            for (int32_t k = v0 + 4 * (int32_t)threadIdx.x; k < v1; k += 4 * ORDER_NT) {
-                const int4 v = *reinterpret_cast<const int4 *>(l.perm + k);
-                set(v.x), set(v.y), set(v.z), set(v.w);
-            }
-            if (s0 + (int32_t)threadIdx.x < v0) set(l.perm[s0 + threadIdx.x]);
-            if (v1 + (int32_t)threadIdx.x < s1) set(l.perm[v1 + threadIdx.x]);
-            __syncthreads();
-            uint32_t b[PER];
-            int n = 0;
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                b[q] = bits[PER * threadIdx.x + q];
-                n += __popc(b[q]);
-            }
-            const int incl = wave_incl_scan(n);
-            if (lane == 63) s_tot[wid] = incl;
-            __syncthreads();
-            int32_t to = at + incl - n;
-#pragma unroll
-            for (int w = 0; w < ORDER_NT / 64; w++) {
-                to += w < wid ? s_tot[w] : 0;
-                at += s_tot[w];
-            }
-#pragma unroll
-            for (int q = 0; q < PER; q++)
-                for (uint32_t m = b[q]; m; m &= m - 1)
-                    l.rank[to++] = (int32_t)first + 32 * (PER * (int32_t)threadIdx.x + q) + __ffs(m) - 1;
-            __syncthreads();  // bits and sums are read, the ranks written
+        for (int32_t k = v0 + 4 * (int32_t)threadIdx.x; k < v1; k += 4 * ORDER_NT) {
+            const int4 v = *reinterpret_cast<const int4 *>(l.perm + k);
+            set(v.x), set(v.y), set(v.z), set(v.w);
         }
-        for (int32_t k = s0 + (int32_t)threadIdx.x; k < s1; k += ORDER_NT) l.perm[k] = l.rank[k];
+        if (s0 + (int32_t)threadIdx.x < v0) set(l.perm[s0 + threadIdx.x]);
+        if (v1 + (int32_t)threadIdx.x < s1) set(l.perm[v1 + threadIdx.x]);
+        const int smaller = wave_incl_scan(before);
+        if (lane == 63) s_before[wid] = smaller;
+        __syncthreads();
+        uint32_t b[PER];
+        int n = 0;
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            b[q] = bits[PER * threadIdx.x + q];
+            n += __popc(b[q]);
+        }
+        const int incl = wave_incl_scan(n);
+        if (lane == 63) s_tot[wid] = incl;
+        __syncthreads();
+        int32_t to = s0 + incl - n;
+#pragma unroll
+        for (int w = 0; w < ORDER_NT / 64; w++) to += s_before[w] + (w < wid ? s_tot[w] : 0);
+#pragma unroll
+        for (int q = 0; q < PER; q++)
+            for (uint32_t m = b[q]; m; m &= m - 1)
+                l.rank[to++] = (int32_t)first + 32 * (PER * (int32_t)threadIdx.x + q) + __ffs(m) - 1;
+        __syncthreads();  // bits and sums are read
     }
 }
 
@@ -300,11 +315,12 @@ int bin_lists(vpbs_ctx *c, SortBuffers &sb, BinList *lists, int count, hipStream
         g.geom.G[d] = c->G[d];
         g.geom.scale[d] = (double)c->G[d] / c->p.Ls[d];
     }
-    int64_t n = 0, nsum = 0, nlarge = 0;  // nlarge: at most
+    int64_t n = 0, nsum = 0, nlarge = 0, nmax = 0;  // nlarge: at most
     for (int t = 0; t < count; t++) {
         n += lists[t].n;
         nsum += sums_size(lists[t].nbins + 1);
         if (lists[t].order_large && bin_large(lists[t].n, lists[t].n)) nlarge += lists[t].n / (BIN_LARGE + 1);
+        nmax = std::max(nmax, lists[t].n);
     }
     VPBS_TRY(grow(c, &sb.rank, &sb.cap_n, n));
     VPBS_TRY(grow(c, &sb.sums, &sb.cap_sums, nsum));
@@ -339,7 +355,10 @@ int bin_lists(vpbs_ctx *c, SortBuffers &sb, BinList *lists, int count, hipStream
         }
     bin_scan<<<tb, SCAN_BS, 0, s>>>(g, deep);
     bin_scatter<<<eb, 256, 0, s>>>(g);
-    if (nlarge) bin_order<<<(unsigned)std::min(nlarge, ORDER_BLOCKS), ORDER_NT, 0, s>>>(g);
+    if (nlarge) {
+        const int64_t windows = (nmax + ORDER_WINDOW - 1) / ORDER_WINDOW;
+        bin_order<<<(unsigned)std::min(nlarge * windows, ORDER_BLOCKS), ORDER_NT, 0, s>>>(g, (int)windows);
+    }
     VPBS_HIP(c, hipGetLastError());
     return VPBS_OK;
 }

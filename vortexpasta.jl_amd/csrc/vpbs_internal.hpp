@@ -42,14 +42,15 @@ constexpr int SPREAD_TX = 16, SPREAD_TY = 8, SPREAD_TZ = 8;
 // A list of positions to bin (sort.hip): by cell of the short-range cell lists, or by the
 // spreading tile or the slab of the first stencil cell.
 enum BinKind { BIN_CELL, BIN_TILE, BIN_SLAB };
-// Whether a bin of a list of n elements is put in order by a block of its own (bin_order in sort.hip) and
-// not by counting. Sort and records of one bin of 600 points and nodes take 52 µs so and 47 by counting,
-// of 1000 56 and 62, of 2000 62 and 91, of 8000 70 and 277. In short lists counting costs at most 0.5 ms
-// (all elements in one bin), and the launch, 5 µs of every call, is left out.
+// Whether a bin of a list of n elements is put in order by blocks of its own (bin_order in sort.hip) and
+// not by counting. Sort and records of one bin of 600 points and nodes take 55 µs so and 47 by counting,
+// of 1000 55 and 62, of 2000 54 and 91, of 8000 62 and 277; a bin costs a pass over it for every window of
+// 131072 indices of the list, hence the bound that grows with n^1/2. In short lists counting costs at most
+// 0.5 ms (all elements in one bin), and the launch, 5 µs of every call, is left out.
 constexpr int BIN_LARGE = 768;
 constexpr int64_t BIN_SHORT_LIST = 16384;
 __host__ __device__ constexpr bool bin_large(int64_t n, int64_t population) {
-    return n > BIN_SHORT_LIST && population > BIN_LARGE;
+    return n > BIN_SHORT_LIST && population > BIN_LARGE && 4 * population * population > n;
 }
 struct BinList {
     int kind;
@@ -59,8 +60,9 @@ struct BinList {
     int32_t *start;     // out: start[b] = first place of bin b, start[nbins] = n
     int32_t *perm;      // out: the elements of every bin, in any order inside it
     int32_t *cell;      // out, or null: per element (ix, iy, iz, key) of its cell
-    bool order_large;   // large bins in order of index
-    int32_t *rank = nullptr, *sums = nullptr;  // scratch
+    bool order_large;   // large bins in order of index, in rank
+    int32_t *rank = nullptr;  // scratch, then the elements of large bins in order, at the bin's places
+    int32_t *sums = nullptr;  // scratch
 };
 struct BinGeom {
     Box box;
