@@ -31,16 +31,25 @@ def run(fake_hip, scenario, *args):
 
 @pytest.mark.parametrize("work", ["points", "advance", "learned", "gradient"])
 def test_out_of_memory_while_growing(fake_hip, work):
-    """Buffers grow for a larger call and one allocation after the other fails: that call says so, no call after it
-    takes the freed buffers for valid ones, and a smaller call then has every buffer that it has in a new context."""
+    """Buffers grow for a larger call and one allocation after the other fails: that call says so or does without, no
+    call after it takes the freed buffers for valid ones, and a smaller call then has every buffer that it has in a new
+    context."""
     out = run(fake_hip, work)
     assert out["allocations"] >= 3
     for k, after in enumerate(out["after"], 1):
-        assert after["refused"], f"allocation {k}: the larger call did not fail"
+        assert after["refused"] or after["grid"], f"allocation {k}: the larger call did not fail"
         assert not after["stale"], f"allocation {k}: {after['stale']} took freed buffers"
         assert not after["again"], f"allocation {k}: the smaller call: {after['again']}"
         assert len(after["blocks"]) == len(out["fresh"]), f"allocation {k}: buffers missing"
         assert all(a >= b for a, b in zip(after["blocks"], out["fresh"])), f"allocation {k}: buffers too small"
+
+
+def test_interpolation_without_memory_for_slabs(fake_hip):
+    """The six buffers of the interpolation fused with the inverse x transform: without one of them a call interpolates
+    from the real grid, which took less memory all along, and with memory again the next one is fused again."""
+    out = run(fake_hip, "points")
+    assert [a["grid"] for a in out["after"]].count(True) == 6
+    assert all(a["fused_again"] for a in out["after"])
 
 
 @pytest.mark.parametrize("call", ["hipHostGetDevicePointer", "hipLaunchKernel"])
@@ -133,9 +142,9 @@ def grow_and_fail(vp, fake, kind):
     s = w.start()
     w.call(s, small)
     fresh = blocks()
-    before = fake.fake_mallocs()
+    before, grids = fake.fake_mallocs(), fake.fake_launches(b"spec_x_inverse")
     w.call(s, large)
-    count = fake.fake_mallocs() - before
+    count, ordinary = fake.fake_mallocs() - before, fake.fake_launches(b"spec_x_inverse") - grids
     s.close()
     if hasattr(s, "net"):
         s.net.close()
@@ -145,21 +154,24 @@ def grow_and_fail(vp, fake, kind):
         s = w.start()
         w.call(s, small)
         fake.fake_fail_malloc(k)
+        grids = fake.fake_launches(b"spec_x_inverse")
         try:
             w.call(s, large)
             refused = False
         except vp._lib.VpbsError as e:
             refused = "out of memory" in str(e)
         fake.fake_fail_malloc(0)
+        grid = not refused and fake.fake_launches(b"spec_x_inverse") - grids > ordinary
         # what a failed set_points or set_filaments leaves; later stages may fail with the points in place
         pts = ctypes.c_int(s._L.vpbs_get_points(s._h, *([None] * 8))).value == 0 if kind != "gradient" else True
         stale = [] if pts else w.stale(s)
-        again = ""
+        again, slabs = "", fake.fake_launches(b"x_inverse_interp")
         try:
             w.call(s, small)
         except vp._lib.VpbsError as e:
             again = str(e)
-        out["after"].append({"refused": refused, "stale": stale, "again": again, "blocks": blocks()})
+        out["after"].append({"refused": refused, "grid": grid, "stale": stale, "again": again, "blocks": blocks(),
+                             "fused_again": fake.fake_launches(b"x_inverse_interp") > slabs})
         s.close()
         if hasattr(s, "net"):
             s.net.close()
@@ -191,7 +203,7 @@ def main():
     fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
     fake.fake_mallocs.restype = fake.fake_launches.restype = ctypes.c_long
     fake.fake_fail_malloc.argtypes = [ctypes.c_long]
-    fake.fake_fail_call.argtypes = [ctypes.c_char_p]
+    fake.fake_fail_call.argtypes = fake.fake_launches.argtypes = [ctypes.c_char_p]
     sys.path.insert(0, str(HERE.parent))
     import __graft_entry__ as ge
 

@@ -983,26 +983,43 @@ int inverse_to_grid(vpbs_ctx *c, Cx<CT> *zp) {
     return VPBS_OK;
 }
 
-// Node buffers of the slab interpolation, grown with Np.
-int slab_node_buffers(vpbs_ctx *c) {
+// Node buffers of the slab interpolation, grown with Np (its partial sums alone take up to 1.9 KB a node).
+// fit = false: the GPU has no memory for them, and the interpolation goes through the real grid, which
+// needs none.
+int slab_node_buffers(vpbs_ctx *c, bool &fit) {
     const int64_t Np = c->Np;
+    fit = true;
     if (Np <= c->cap_nd) return VPBS_OK;
     c->cap_nd = 0;  // until all of them are there
-    void **bufs[] = {(void **)&c->nd_key, (void **)&c->nd_perm, (void **)&c->nd_i0, (void **)&c->nd_node,
-                     &c->nd_rec, &c->slab_part};
-    for (void **b : bufs)
-        if (*b) {
-            VPBS_HIP(c, hipFree(*b));
-            *b = nullptr;
+    const size_t es = c->p.precision == VPBS_F32 ? sizeof(float) : sizeof(double), i4 = sizeof(int32_t);
+    const struct {
+        void **p;
+        size_t bytes;  // per node
+    } bufs[] = {{(void **)&c->nd_key, i4},
+                {(void **)&c->nd_perm, i4},
+                {(void **)&c->nd_i0, 3 * i4},
+                {(void **)&c->nd_node, i4},
+                {&c->nd_rec, es * (size_t)slab_rec_len(2 * c->p.nufft_m, (int)es)},
+                {&c->slab_part, es * 3 * (size_t)spectral_slab_slots(c)}};
+    auto drop = [&]() -> int {
+        for (const auto &b : bufs)
+            if (*b.p) {
+                VPBS_HIP(c, hipFree(*b.p));
+                *b.p = nullptr;
+            }
+        return VPBS_OK;
+    };
+    VPBS_TRY(drop());
+    for (const auto &b : bufs) {
+        const hipError_t e = hipMalloc(b.p, b.bytes * (size_t)Np);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();  // handled here
+            *b.p = nullptr;
+            fit = false;
+            return drop();
         }
-    const size_t es = c->p.precision == VPBS_F32 ? sizeof(float) : sizeof(double);
-    const size_t rec = (size_t)slab_rec_len(2 * c->p.nufft_m, (int)es);
-    VPBS_HIP(c, hipMalloc((void **)&c->nd_key, sizeof(int32_t) * (size_t)Np));
-    VPBS_HIP(c, hipMalloc((void **)&c->nd_perm, sizeof(int32_t) * (size_t)Np));
-    VPBS_HIP(c, hipMalloc((void **)&c->nd_i0, sizeof(int32_t) * 3 * (size_t)Np));
-    VPBS_HIP(c, hipMalloc((void **)&c->nd_node, sizeof(int32_t) * (size_t)Np));
-    VPBS_HIP(c, hipMalloc(&c->nd_rec, es * rec * (size_t)Np));
-    VPBS_HIP(c, hipMalloc(&c->slab_part, es * 3 * (size_t)spectral_slab_slots(c) * (size_t)Np));
+        VPBS_HIP(c, e);
+    }
     c->cap_nd = Np;
     return VPBS_OK;
 }
@@ -1016,16 +1033,17 @@ int launch_lr(vpbs_ctx *c, uint32_t flags) {
     const CT beta = (CT)c->es_beta;
 
     stage_begin(c, ST_LRSORT, s);
-    if (c->slab_interp) VPBS_TRY(slab_node_buffers(c));
+    bool slab = c->slab_interp;
+    if (slab) VPBS_TRY(slab_node_buffers(c, slab));
     BinList lists[2] = {
         {BIN_TILE, Nq, c->ntiles, c->points, c->lr_key, c->lr_start, c->lr_perm, nullptr, true},
         {BIN_SLAB, Np, c->nslabs, c->nodes, c->nd_key, c->nd_start, c->nd_perm, nullptr, true},
     };
-    VPBS_TRY(bin_lists(c, c->sort_lr, lists, c->slab_interp ? 2 : 1, s));
+    VPBS_TRY(bin_lists(c, c->sort_lr, lists, slab ? 2 : 1, s));
     GatherArgs<CT> ga{g, beta, Nq, Np, nblocks(Nq, 256), c->lr_key, c->lr_start, c->lr_perm, lists[0].rank, c->nd_key,
-                      c->nd_start, c->nd_perm, lists[1].rank, c->points, c->charges, c->nodes, c->lr_i0, c->nd_i0, c->nd_node, (CT *)c->lr_w,
-                      (CT *)c->nd_rec};
-    launch_gather<CT>(ga, ga.point_blocks + (c->slab_interp ? nblocks(Np, 256) : 0), s);
+                      c->nd_start, c->nd_perm, lists[1].rank, c->points, c->charges, c->nodes, c->lr_i0, c->nd_i0,
+                      c->nd_node, (CT *)c->lr_w, (CT *)c->nd_rec};
+    launch_gather<CT>(ga, ga.point_blocks + (slab ? nblocks(Np, 256) : 0), s);
     stage_end(c, ST_LRSORT, s);
 
     CT *grid = (CT *)c->grid;
@@ -1044,17 +1062,17 @@ int launch_lr(vpbs_ctx *c, uint32_t flags) {
         // inverse transforms to the nodes: with slab interpolation the inverse x transform
         // runs inside the interpolation kernel (the real grid is not written)
         stage_begin(c, ST_FFTB, s);
-        if (vel) VPBS_TRY(c->slab_interp ? spectral_y_inverse(c, c->zpen) : spectral_inverse(c, c->zpen));
+        if (vel) VPBS_TRY(slab ? spectral_y_inverse(c, c->zpen) : spectral_inverse(c, c->zpen));
         stage_end(c, ST_FFTB, s);
         stage_begin(c, ST_INTERP, s);
         if (vel) {
-            if (c->slab_interp)
+            if (slab)
                 VPBS_TRY(spectral_x_inverse_interp(c, c->v_lr));
             else
                 launch_interp<CT>(g, Np, c->nodes, beta, grid, c->v_lr, s);
         }
         if (psi) {
-            if (c->slab_interp) {
+            if (slab) {
                 VPBS_TRY(spectral_y_inverse(c, c->zpen2));
                 VPBS_TRY(spectral_x_inverse_interp(c, c->psi_lr));
             } else {
