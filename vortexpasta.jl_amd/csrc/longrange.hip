@@ -61,12 +61,10 @@ constexpr int MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
 double *g_scratch_ptr[MAX_DEVICES] = {};  // device address of `scratch` on each GPU (null: not taken yet)
 
-
 // Spreading tile: 16 × 8 × 8 cells: 16 x-cells are the columns and 16 rows (8 in y,
 // 2 in z) the rows of a 16×16 matrix-core tile, 4 of them and 3 components in 48
 // (FP32) or 96 (FP64) accumulator registers.
 constexpr int TX = SPREAD_TX, TY = SPREAD_TY, TZ = SPREAD_TZ;
-constexpr int MAXM = 8;     // largest supported half-support
 
 inline unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -100,12 +98,6 @@ struct LRGeom {
 // along x, y and z, then the 3 charge components, padded to 16 bytes.
 constexpr int rec_len(int W) { return (3 * W + 3 + 3) & ~3; }
 
-// Position of real grid value (x, y, z) of one component: rows y = 2p and
-// y = 2p + 1 are interleaved as the real and imaginary parts of complex row p.
-__device__ inline int64_t gidx(const LRGeom &g, int x, int y, int z) {
-    return (((int64_t)z * (g.G[1] >> 1) + (y >> 1)) * g.G[0] + x) * 2 + (y & 1);
-}
-
 template <typename CT>
 struct alignas(2 * sizeof(CT)) Cx {
     CT re, im;
@@ -119,7 +111,7 @@ struct alignas(2 * sizeof(CT)) Cx {
 // weights φ((i0_d + k - u_d)/m) per direction and the charge, computed once
 // here instead of once per tile in the spreading kernel.
 // Records are rec_len(W) values (a multiple of 16 bytes) moved with 16-byte vector
-// accesses: one thread writes or reads a whole record.
+// accesses: one thread writes a whole record.
 template <typename CT, int N>
 __device__ __forceinline__ void store_rec(CT *__restrict__ p, const CT (&r)[N]) {
     static_assert((N * sizeof(CT)) % 16 == 0, "records are whole 16-byte vectors");
@@ -129,22 +121,6 @@ __device__ __forceinline__ void store_rec(CT *__restrict__ p, const CT (&r)[N]) 
     } else {
 #pragma unroll
         for (int k = 0; k < N; k += 2) reinterpret_cast<double2 *>(p)[k / 2] = double2{r[k], r[k + 1]};
-    }
-}
-template <typename CT, int N>
-__device__ __forceinline__ void load_rec(const CT *__restrict__ p, CT (&r)[N]) {
-    if constexpr (sizeof(CT) == 4) {
-#pragma unroll
-        for (int k = 0; k < N; k += 4) {
-            const float4 v = reinterpret_cast<const float4 *>(p)[k / 4];
-            r[k] = v.x, r[k + 1] = v.y, r[k + 2] = v.z, r[k + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < N; k += 2) {
-            const double2 v = reinterpret_cast<const double2 *>(p)[k / 2];
-            r[k] = v.x, r[k + 1] = v.y;
-        }
     }
 }
 

@@ -614,7 +614,6 @@ int point_data_from_state(vpbs_ctx *c, bool uploaded) {
         qd.lim_p[1] = g;
     }
     c->have_points = false;
-    c->stage_ran[ST_POINTS] = false;
     stage_break(c, s);
     stage_begin(c, ST_POINTS, s);
     auto *flag = reinterpret_cast<volatile unsigned int *>(c->host_stage);

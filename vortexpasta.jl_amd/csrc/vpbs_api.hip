@@ -36,17 +36,15 @@ int fail(vpbs_ctx *c, int code, const char *fmt, ...) {
 // Stages are timed by events without a system-scope fence (nothing but their times is read from
 // them), and a stage that follows another on its stream starts from that one's end event: a pair of
 // fencing events around every stage held the next stage up by 7 µs, one of these by 1 (10 stages of
-// one kernel each: 456 and 397 µs, without events 387).
+// one kernel each: 456 and 397 µs, without events 387). A stage runs at most once in a call: the end
+// events that others start from are recorded once.
 void stage_begin(vpbs_ctx *c, Stage st, hipStream_t s) {
-    const hipEvent_t after = c->stage_after[s == c->s_lr];
-    // a stage that runs again (second field) has an event of its own: the end event it would start
-    // from is recorded again as well
-    if (after && !c->stage_ran[st]) {
-        c->stage_from[st] = after;
-    } else {
-        (void)hipEventRecord(c->ev_beg[st], s);
-        c->stage_from[st] = c->ev_beg[st];
+    hipEvent_t from = c->stage_after[s == c->s_lr];
+    if (!from) {
+        from = c->ev_beg[st];
+        (void)hipEventRecord(from, s);
     }
+    c->stage_from[st] = from;
     c->stage_ran[st] = true;
 }
 
