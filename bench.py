@@ -528,10 +528,13 @@ def main():
     log(f"end to end: {json.dumps(e2e)}")
 
     # roofline of the dominant long-range kernel of the FP32 path (our own kernels only); the
-    # hand-written transforms take the inverse x transform into the interpolation on the x-grids
-    # that the configurations have
+    # hand-written transforms take the inverse x transform into the interpolation, and the z
+    # transforms into registers, on the grid lengths compiled for it
     fused = args.fft == "fused"
-    slab = fused and grid[0] in (96, 192, 384, 768, 1536)
+    compiled = (32, 64, 96, 128, 160, 192, 256, 288, 320, 384, 512, 576, 640, 768, 1024, 1152, 1536)
+    slab = fused and grid[0] in compiled and grid[0] != 1152
+    z_kernel = (f"spec_z_reg<float, {grid[2]}, true, false>" if grid[2] in compiled
+                else f"spec_z_fourier<float, {grid[2] if grid[2] in (480, 960) else 0}>")
     lr_kernels = ["spread", "fourier", "interp"]
     dom = max(lr_kernels, key=lambda k: st32.get(k, 0.0))
     nbytes = stage_bytes(dom, 4, grid, spl.Ns, pd.Np, pd.Nq, slab)
@@ -540,7 +543,7 @@ def main():
                  for k in ("spread", "fft_forward", "fourier", "fft_backward", "interp") if st32.get(k, 0) > 0}
 
     kname = {"spread": f"spread_tiles_kernel<float, {2 * args.m}>",
-             "fourier": f"spec_z_reg<float, {grid[2]}, true, false>" if fused or args.fft == "separate" else "fourier_kernel<float>",
+             "fourier": z_kernel if fused or args.fft == "separate" else "fourier_kernel<float>",
              "interp": f"x_inverse_interp<float, {2 * args.m}, {grid[0]}>" if slab
              else f"interp_kernel_wave<float, {2 * args.m}>"}[dom]
     # the same stages with each range alone (the other stream idle): what the kernels reach by

@@ -41,8 +41,9 @@ extern "C" {
 
 /* transforms of the long-range part (vpbs_params.fft) */
 #define VPBS_FFT_FUSED 0    /* hand-written FFTs fused with the pencil reorderings and the Fourier-space kernel;
-                               on x-grids of up to 1536 cells (lengths 2^a·3^b and 2^a·5^b) also the inverse x
-                               transform fused with the interpolation (no real grid written on that side) */
+                               on x-grids of up to 768 cells whose length has not both factors 3 and 5, of 1024
+                               and of 1536 cells also the inverse x transform fused with the interpolation (no
+                               real grid written on that side), if the GPU has memory for its node buffers */
 #define VPBS_FFT_ROCFFT 1   /* rocFFT 1D transforms with separate reordering and Fourier-space kernels */
 #define VPBS_FFT_SEPARATE 2 /* the hand-written FFTs of VPBS_FFT_FUSED with the interpolation in a kernel of its own */
 
@@ -88,7 +89,8 @@ typedef struct vpbs_params {
                               z > 3072 / 1536) use rocFFT */
 } vpbs_params;
 
-/* Per-stage GPU times of the last vpbs_compute, in milliseconds (HIP events). */
+/* Per-stage GPU times of the last vpbs_compute, in milliseconds (HIP events). A stage runs from the end of the
+   stage before it on its stream, so a wait between them (for the host, say) counts to it. */
 typedef struct vpbs_timings {
     double total;        /* whole compute, host wall-clock (includes waits) */
     double local_term;   /* LIA kernel */

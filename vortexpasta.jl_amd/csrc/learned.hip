@@ -641,7 +641,6 @@ __global__ void correction_apply(int64_t Np, const float *__restrict__ y, const 
     }
 }
 
-// Sums over the sample of |Δv_pred − Δv|², |Δv|² and |v_cheap + Δv|² (fixed-order tree).
 // Per-block partial sums (grid-stride, at most CHK_NV blocks) of the squared errors of the corrected
 // and of the cheap velocity over the sample, and of |v|² over every node, added by check_reduce's
 // fixed tree (one partial per thread). The sample over all blocks: one block that walked it alone
@@ -675,7 +674,10 @@ __global__ __launch_bounds__(256) void check_partial(int64_t Np, const double *_
     if (threadIdx.x < 3) part[threadIdx.x * CHK_NV + blockIdx.x] = red[threadIdx.x][0];
 }
 
-// out: both squared errors of the sample, and |v|² of the field scaled to the sample's size.
+// out = (Σ_s |Δv_pred − Δv|², Σ_s |Δv|², (ns/Np)·Σ_all |v|²) over the sample s: the ratios of the first two to
+// the third estimate the squared relative L2 errors of the corrected and the cheap velocity over the whole
+// field. (Normalising by the sample's own Σ|v|² would not: a few fast nodes hold much of the field's Σ|v|²,
+// and a 1 % sample that misses them overstates the relative error two- to four-fold.)
 __global__ __launch_bounds__(1024) void check_reduce(int64_t Np, int64_t ns, const double *__restrict__ part, int nb,
                                                      double *__restrict__ out) {
     __shared__ double red[3][1024];

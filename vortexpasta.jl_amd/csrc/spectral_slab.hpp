@@ -318,7 +318,8 @@ __global__ void slab_reduce(int64_t Np, int nslot, const CT *__restrict__ part, 
     out[c * Np + i] = acc;
 }
 
-// The compiled lengths: those that reg_plan covers and whose slab fits the LDS and a block.
+// The compiled lengths: every grid length (32·2^a·3^b·5^c) up to 768 that reg_plan covers, 1024 and 1536
+// (800, 864, 1152 and 1280 cells interpolate from the real grid).
 #define SLAB_LENGTHS(F)                                                                             \
     F(32) F(64) F(96) F(128) F(160) F(192) F(256) F(288) F(320) F(384) F(512) F(576) F(640) F(768) \
     F(1024) F(1536)
